@@ -1,5 +1,5 @@
-"""The fast projectors' split of values over the whole float32 range: images and planograms whose rows hold
-values 2^-36 to 2^-120 apart.
+"""The fast projectors' split of values and weights over the whole float32 range: images and planograms whose rows hold
+values 2^-36 to 2^-120 apart, and outputs that only a small interpolation weight reaches.
 
 Tolerance.  Beside a hot value the cold outputs are the same products as without it, and an image is the sum of its parts,
 so only the order and the rounding of the sums may differ: 2^-24 each, at most 5 per block of 4 inner indices and 3 per v1
@@ -11,6 +11,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
+from petl_amd.petl_server import PETLserver  # noqa: E402
 from test_gpu_back_tiles import back  # noqa: E402
 from test_gpu_forward_tiles import CASES, TOL, forward, make, rel  # noqa: E402
 
@@ -85,3 +86,33 @@ def test_ramp_planogram(oracle, top, step, mode):
     on = ref > 0
     f = back(s, g).astype(np.float64)
     assert np.max(np.abs(f[on] / ref[on] - 1.0)) < ETOL
+
+
+@pytest.mark.parametrize("k", [12, 16, 20, 24])
+def test_small_weights(oracle, k):
+    """One voxel up to 2^-k of a bin beside a bin's centre, by another part of it in every view: the bins that get the small
+    part hold it to float32 accuracy (fewer than 10 roundings; the smallest weight, 2^-28, is the rest of a float64 position
+    near 14 bins, which is good to 2^-50 and so to 2^-22 of it)."""
+    s = PETLserver()
+    s.print_warnings = False
+    args = (0.0, 30.0, 20.0, 8.0, 2.0, 1.0, 0.2)
+    s.add_planogram(*args)
+    offs = (1.0, float(np.float32(1.3 * 2.0 ** (1 - k))), 0.7)  # bin centres are odd millimetres; y offset x v0 beside them
+    s.set_volume(1, 1, 1, 2.0, 0.0, *offs)
+    assert s.uses_fast_path(0)
+    plan = oracle.planogram(*args)
+    vol = oracle.volume(1, 1, 1, 2.0, 0.0, *offs)
+    ref = oracle.project([plan], vol, np.full((1, 1, 1), 0.7), dtype=np.float64)[0]
+    g = forward(s, plan, np.full((1, 1, 1), 0.7)).astype(np.float64)
+    small = (ref > 0) & (ref < 4.0 * 2.0 ** -k)
+    small[:, :plan.shape[1] // 2 + 1] = False  # on this side the small weight is one minus a float, no better than 2^-25
+    assert small.sum() > 20
+    assert np.max(np.abs(g[small] / ref[small] - 1.0)) < 10 * 2.0 ** -24
+    iv1, iv0, iu1, iu0 = (int(x[-1]) for x in np.nonzero(small))
+    for mode in ("petl", "matched"):
+        s.set_backprojector_mode(mode)
+        y = np.zeros(plan.shape, np.float32)
+        y[iv1, iv0, iu1, iu0] = 0.3
+        refb = oracle.backproject([plan], vol, [y.astype(np.float64)], mode=mode, dtype=np.float64)
+        assert refb[0, 0, 0] > 0
+        assert abs(back(s, y)[0, 0, 0].astype(np.float64) / refb[0, 0, 0] - 1.0) < 10 * 2.0 ** -24
