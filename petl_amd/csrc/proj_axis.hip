@@ -131,6 +131,8 @@ __global__ void __launch_bounds__(64 * AX_WAVES) axis_fwd_kernel(float* __restri
             }
         }
     }
+    static_assert(AX_NI * AX_R <= 32, "a bit per bin of a lane");
+    unsigned again = 0;
 #pragma unroll
     for (int j = 0; j < AX_NI; j++) {
         const int item = item0 + j;
@@ -142,9 +144,39 @@ __global__ void __launch_bounds__(64 * AX_WAVES) axis_fwd_kernel(float* __restri
             for (int r = 0; r < AX_R; r++)
                 if (iu1_0 + r < P.Nu1) {
                     const int64_t gi = ((int64_t(iv1) * P.Nv0 + v) * P.Nu1 + iu1_0 + r) * P.Nu0 + iu0;
-                    g[gi] = gen_epilogue(in && live[r] ? acc[j][r] * scale : 0.0f, gi, epilogue, y, resp, wts);
+                    if (in && live[r] && !__builtin_isfinite(acc[j][r]))
+                        again |= 1u << (j * AX_R + r);
+                    else
+                        g[gi] = gen_epilogue(in && live[r] ? acc[j][r] * scale : 0.0f, gi, epilogue, y, resp, wts);
                 }
         }
+    }
+    // A cell beside the footprint has the weight zero, which an infinity or a NaN would turn into a NaN: a bin that came out
+    // as one is summed again, over the cells that it meets.
+    const int64_t sk = int64_t(Ns) * Na;
+    for (; again; again &= again - 1) {
+        const int b = __ffs(again) - 1, item = item0 + b / AX_R, v = item / nc, iu0 = (item - v * nc) * 64 + lane;
+        const int iu1 = iu1_0 + b % AX_R;
+        float sum = 0.0f;
+        for (int s = 0; s < Ns; s++) {
+            const float xi = fmaf(A.Au, float(iu0), A.G.xi0[int64_t(v) * A.G.Nsmax + s]);
+            const float c = cross_z(Bz, fmaf(wm.Bs, float(s), wm.Z0), iu1);
+            const int i0 = int(floorf(xi + (0.5f - A.hb)));
+            const int klo = max(0, int(floorf(c - hz + 0.5f))), khi = min(Nz - 1, int(ceilf(c + hz - 0.5f)));
+            for (int a = max(i0, 0); a < min(i0 + NA, Na); a++) {
+                const float w = overlap(xi, A.hb, float(a));
+                float h = 0.0f;
+                for (int k = klo; k <= khi && w > 0.0f; k++) {
+                    const float wz = overlap(c, hz, float(k));
+                    if (wz > 0.0f)
+                        h += vol[int64_t(k) * sk + int64_t(s) * Na + a] * wz;
+                }
+                if (w > 0.0f)
+                    sum += w * h;
+            }
+        }
+        const int64_t gi = ((int64_t(iv1) * P.Nv0 + v) * P.Nu1 + iu1) * P.Nu0 + iu0;
+        g[gi] = gen_epilogue(sum * A.G.views[int64_t(iv1) * P.Nv0 + v].scale, gi, epilogue, y, resp, wts);
     }
 }
 
@@ -170,8 +202,8 @@ __global__ void __launch_bounds__(256) axis_back_u0_kernel(const float* __restri
     for (int r = 0; r < AX_RB; r++)
         acc[r] = 0.0f;
     const GenView* wr = A.G.views + int64_t(iv1) * P.Nv0;
-    for (int iv0 = 0; iv0 < P.Nv0; iv0++) {
-        float w[NP];
+    // the column's bins in view iv0, p0 ... p0 + NP - 1, and their weights (zero outside its footprint)
+    auto weights = [&](int iv0, float(&w)[NP]) {
         int p0;
         if (MATCHED) {
             // bins whose footprint meets cell a: crossings within hb + 1/2 of it (one bin of margin below)
@@ -190,13 +222,45 @@ __global__ void __launch_bounds__(256) axis_back_u0_kernel(const float* __restri
             for (int k = 0; k < NP; k++)
                 w[k] = fmaxf(0.0f, fminf(float(p0 + k) + 0.5f, B0) - fmaxf(float(p0 + k) - 0.5f, A0)) * wr[iv0].lpetl;
         }
-        const float* gv = g + ((int64_t(iv1) * P.Nv0 + iv0) * P.Nu1 + iu1_0) * P.Nu0;
+        return p0;
+    };
+    const float* g1 = g + (int64_t(iv1) * P.Nv0 * P.Nu1 + iu1_0) * P.Nu0;
+    for (int iv0 = 0; iv0 < P.Nv0; iv0++) {
+        float w[NP];
+        const int p0 = weights(iv0, w);
+        const float* gv = g1 + int64_t(iv0) * P.Nu1 * P.Nu0;
 #pragma unroll
         for (int r = 0; r < AX_RB; r++) {
             const float* q = gv + unsigned(min(r, rmax)) * rowb + unsigned(p0);
 #pragma unroll
             for (int k = 0; k < NP; k++)
                 acc[r] += w[k] * q[k];
+        }
+    }
+    // A bin beside the footprint has the weight zero, which an infinity or a NaN would turn into a NaN: columns that come out
+    // as one are summed again, over the bins that they meet.
+    bool void_row = false;
+#pragma unroll
+    for (int r = 0; r < AX_RB; r++)
+        void_row = void_row || !__builtin_isfinite(acc[r]);
+    if (void_row) {
+#pragma unroll
+        for (int r = 0; r < AX_RB; r++)
+            acc[r] = 0.0f;
+#pragma unroll 1
+        for (int iv0 = 0; iv0 < P.Nv0; iv0++) {
+            float w[NP];
+            const int p0 = weights(iv0, w);
+            const float* gv = g1 + int64_t(iv0) * P.Nu1 * P.Nu0;
+#pragma unroll
+            for (int r = 0; r < AX_RB; r++) {
+                const float* q = gv + unsigned(min(r, rmax)) * rowb + unsigned(p0);
+#pragma unroll
+                for (int k = 0; k < NP; k++) {
+                    const float x1 = w[k] > 0.0f ? q[k] : 0.0f;
+                    acc[r] += w[k] * x1;
+                }
+            }
         }
     }
     if (col < ncol) {
