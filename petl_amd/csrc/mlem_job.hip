@@ -37,14 +37,16 @@ constexpr int UP_CHUNKS = 3, UP_THREADS = 8;
 
 namespace {
 
-bool page_locked(const void* h)
+// whether HIP knows the memory, page-locked, managed or a device's: a plain copy takes any of it, and the threads' copies
+// must not read a device's
+bool known_memory(const void* h)
 {
     hipPointerAttribute_t a{};
     if (hipPointerGetAttributes(&a, h) != hipSuccess) {
-        (void)hipGetLastError();  // (memory that HIP does not know)
+        (void)hipGetLastError();
         return false;
     }
-    return a.type == hipMemoryTypeHost;
+    return a.type != hipMemoryTypeUnregistered;
 }
 
 struct Events {
@@ -66,7 +68,7 @@ struct Events {
 
 void upload(Model& m, void* d, const void* h, size_t n, hipStream_t s)
 {
-    if (n < UP_SMALL || page_locked(h)) {
+    if (n < UP_SMALL || known_memory(h)) {
         h2d(d, h, n, s);
         return;
     }
