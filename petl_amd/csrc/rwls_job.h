@@ -27,6 +27,8 @@ struct RwlsParams {
 class RwlsJob {
 public:
     RwlsJob(Model& m, const RwlsParams& prm);
+    // gives the buffers back if they hold more than the model keeps
+    ~RwlsJob();
     // uploads g (and W, response) and f0 (host arrays), forms the weights, the residual and the
     // preconditioner.  f0 follows the reference's start rules already (negatives clipped when nonneg).
     void setup(float* const* g, const float* f0, bool f0_nonzero, float* const* W, float* const* response,
@@ -48,7 +50,9 @@ private:
     int64_t V_ = 0;
     size_t nP_ = 0;
     std::vector<int64_t> G_;
-    // the model's buffers, kept between calls (MLEM's data, ratio, projection and volumes among them)
+    // the model's buffers (MLEM's data, ratio, projection and volumes among them), kept between calls up to KEEP bytes
+    // (a small reconstruction's allocations are a good part of it, a large one's are not)
+    static constexpr size_t KEEP = size_t(4) << 30;
     std::vector<DevBuf>&g_, &r_, &Pd_, &W_, &resp_;
     DevBuf &f_, &grad_, &u_, &d_, &grad_old_, &Q_, &red_;
     std::vector<float*> gp_, rp_, Pdp_, Wp_, respp_;

@@ -36,6 +36,20 @@ RwlsJob::RwlsJob(Model& m, const RwlsParams& prm)
         G_[i] = m.plans[i].elems();
 }
 
+RwlsJob::~RwlsJob()
+{
+    std::vector<DevBuf*> all = {&f_, &grad_, &u_, &d_, &grad_old_, &Q_, &red_};
+    for (std::vector<DevBuf>* v : {&g_, &r_, &Pd_, &W_, &resp_})
+        for (DevBuf& b : *v)
+            all.push_back(&b);
+    size_t held = 0;
+    for (const DevBuf* b : all)
+        held += b->bytes;
+    if (held > KEEP)
+        for (DevBuf* b : all)
+            b->release();
+}
+
 void RwlsJob::project(const float* x, std::vector<float*>& out, hipStream_t s)
 {
     m_.forward(out.data(), x, EPI_NONE, nullptr, prm_.response ? respp_.data() : nullptr, s);
